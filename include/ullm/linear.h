@@ -90,7 +90,8 @@ typedef uint32_t ullm_linear_encoding_t;
 
 /* How bf16 activations enter the contraction. */
 /* Exact: bf16 activations times dequantized weights, fp32 accumulation.
- * Any M; the decode kernels serve M <= 32 per weight pass. */
+ * Any M; the decode kernels serve M <= 32, block kernels that read each
+ * weight once per block of rows serve more. */
 #define ULLM_LINEAR_ACT_EXACT UINT32_C(0)
 /* Prefill: activations are quantized per token to E4M3 (scale = max|x|/448)
  * and contracted with FP8 weights on the FP8 matrix cores. */
@@ -212,7 +213,8 @@ typedef struct ullm_linear_weight_export_desc_t {
 /* Kernel families reported by ullm_linear_forward_plan. */
 #define ULLM_LINEAR_KERNEL_GEMV UINT32_C(1)        /* decode, bf16 activations */
 #define ULLM_LINEAR_KERNEL_GEMM_DIRECT UINT32_C(2) /* FP8 GEMM, operands from L2 */
-#define ULLM_LINEAR_KERNEL_GEMM_LDS UINT32_C(3)    /* FP8 GEMM, LDS-pipelined */
+#define ULLM_LINEAR_KERNEL_GEMM_LDS UINT32_C(3)    /* activations through LDS: FP8
+                                                    * GEMM, or exact M > 32 */
 
 /* GEMV kernel variants reported by ullm_linear_forward_plan. */
 #define ULLM_LINEAR_GEMV_SINGLE UINT32_C(1)  /* one stripe per workgroup, x from L2 */

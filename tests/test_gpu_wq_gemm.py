@@ -1,0 +1,179 @@
+"""GPU parity of the many-row exact products (gemm_wq.hip): bf16 activations
+times FP8 or AQ4 weights at M > 32, against the C oracle.
+
+The shapes reach every block configuration (checked through
+ullm_linear_forward_plan on a 256-CU device) at the edges where a tile can go
+wrong: rows and columns one past a block, K tails of one to three 128-k steps
+past the pipeline's four, an FP8 K that ends inside a step, K shorter than
+the waves that split it, strided activations, unaligned outputs, and the fused
+epilogues.  Tolerances are the suite's (helpers.assert_close); fp32 outputs
+are also held to 1e-5 of their RMS: sums of at most 4224 fp32 products round
+to about 1e-7, and AQ4's group offset (16 + z against q) raises that by less
+than 30.
+"""
+import numpy as np
+import pytest
+import torch
+
+from helpers import (activations_bf16, assert_close, bf16_tensor_to_f32,
+                     to_torch_bf16, weights)
+
+pytestmark = pytest.mark.gpu
+
+
+def _weight(uh, orc, enc, w, gated=False):
+    if enc == "fp8":
+        enc_w = orc.fp8_quantize_rows(w)
+        return uh.LinearWeight.from_fp8(*enc_w, gated=gated), enc_w
+    enc_w = orc.aq4_quantize(w)
+    return uh.LinearWeight.from_aq4(*enc_w, gated=gated), enc_w
+
+
+def _ref(orc, enc, xb, enc_w):
+    return (orc.fp8_gemv if enc == "fp8" else orc.aq4_gemv)(xb, *enc_w)[0]
+
+
+def _block(lw, x, y, expect):
+    p = lw.plan(x, y)
+    assert p.kernel == 3 and p.split_k == 1, "not a block kernel"
+    if torch.cuda.get_device_properties(x.device).multi_processor_count == 256:
+        assert (p.block_m, p.block_n) == expect, (p.block_m, p.block_n)
+
+
+# (m, n, k): the block on 256 CUs for (fp8, aq4).
+SHAPES = {
+    (87, 40, 128): ((32, 32), (16, 32)),
+    (33, 129, 64): ((32, 32), (16, 32)),
+    (40, 300, 4096): ((16, 32), (16, 32)),
+    (70, 1000, 4224): ((16, 32), (16, 32)),
+    (38, 4106, 384): ((32, 48), (16, 32)),
+    (64, 6000, 2112): ((32, 48), (32, 48)),
+    (38, 6855, 640): ((32, 64), (32, 32)),
+    (48, 6150, 1280): ((32, 64), (32, 64)),
+    (37, 4349, 320): ((32, 48), (16, 32)),
+    (129, 4100, 1280): ((32, 128), (32, 128)),
+    (67, 6318, 2432): ((32, 96), (32, 96)),
+    (38, 9226, 896): ((32, 128), (48, 48)),
+    (34, 9188, 1664): ((48, 48), (48, 48)),
+    (34, 13214, 1792): ((32, 128), (48, 64)),
+    (34, 14658, 2944): ((48, 64), (48, 64)),
+    (1162, 806, 1024): ((64, 64), (32, 64)),
+    (1071, 912, 1152): ((64, 64), (64, 64)),
+    (66, 16580, 256): ((32, 128), (32, 128)),
+    (66, 18300, 320): ((32, 128), (32, 128)),
+    (38, 5732, 384): ((32, 48), (32, 48)),
+    (50, 8524, 2048): ((32, 128), (32, 96)),
+    (38, 18311, 256): ((64, 128), (64, 128)),
+    (38, 16572, 128): ((32, 128), (64, 128)),
+    (200, 24661, 256): ((128, 256), (128, 256)),
+    (67, 22155, 192): ((32, 128), (32, 128)),
+    (321, 27266, 256): ((64, 128), (192, 256)),
+    (387, 23495, 384): ((256, 192), (256, 192)),
+    (385, 23368, 192): ((256, 192), (256, 192)),
+    (257, 16400, 512): ((128, 256), (64, 128)),
+}
+
+
+@pytest.mark.parametrize("m,n,k", list(SHAPES))
+@pytest.mark.parametrize("enc", ["fp8", "aq4"])
+def test_wq_gemm_parity(uh, orc, gpu, enc, m, n, k):
+    if enc == "aq4" and k % 128:
+        pytest.skip("AQ4 K is a multiple of 128")
+    lw, enc_w = _weight(uh, orc, enc, weights(n, k, tag=51))
+    xb = activations_bf16(orc, m, k, tag=m + 400)
+    y_ref = _ref(orc, enc, xb, enc_w)
+    x = to_torch_bf16(xb, gpu)
+    y32 = torch.full((m, n), float("nan"), device=gpu)
+    lw.forward(x, y32)
+    _block(lw, x, y32, SHAPES[(m, n, k)][enc == "aq4"])
+    assert_close(y32.cpu().numpy(), y_ref, rel=1e-5, what=f"{enc} f32 {m}x{n}x{k}")
+    yb = torch.full((m, n), float("nan"), dtype=torch.bfloat16, device=gpu)
+    lw.forward(x, yb)
+    assert_close(bf16_tensor_to_f32(yb), y_ref, bf16_out=True, what=f"{enc} bf16 {m}x{n}x{k}")
+
+
+@pytest.mark.parametrize("m,n", [(50, 1100), (300, 2056)])
+@pytest.mark.parametrize("enc", ["fp8", "aq4"])
+def test_wq_gemm_strided_and_unaligned(uh, orc, gpu, enc, m, n):
+    """x a column slice of a wider buffer whose other columns are NaN, y a
+    column slice at an odd offset (no 16-byte rows), values outside both
+    untouched; a strip block and an 8-wave block."""
+    k = 640
+    lw, enc_w = _weight(uh, orc, enc, weights(n, k, tag=53))
+    xb = activations_bf16(orc, m, k, tag=m + 410)
+    y_ref = _ref(orc, enc, xb, enc_w)
+    wide = torch.full((m, k + 24), float("nan"), dtype=torch.bfloat16, device=gpu)
+    wide[:, 8:8 + k] = to_torch_bf16(xb, gpu)
+    for dt in (torch.bfloat16, torch.float32):
+        buf = torch.full((m, n + 5), 7.0, dtype=dt, device=gpu)
+        y = buf[:, 3:3 + n]
+        lw.forward(wide[:, 8:8 + k], y)
+        assert_close(bf16_tensor_to_f32(y.contiguous()), y_ref, bf16_out=dt == torch.bfloat16,
+                     what=f"{enc} strided")
+        assert torch.all(buf[:, :3] == 7.0) and torch.all(buf[:, 3 + n:] == 7.0)
+
+
+@pytest.mark.parametrize("m,n", [(37, 1040), (300, 2064)])
+@pytest.mark.parametrize("enc", ["fp8", "aq4"])
+@pytest.mark.parametrize("out", [torch.bfloat16, torch.float32])
+def test_wq_gemm_epilogues(uh, orc, gpu, enc, m, n, out):
+    """SiLU-gate (F not a multiple of the block) and an in-place residual,
+    with alpha, in a strip block and an 8-wave block."""
+    k = 384
+    w = weights(n, k, tag=57)
+    xb = activations_bf16(orc, m, k, tag=m + 420)
+    x = to_torch_bf16(xb, gpu)
+    lw, enc_w = _weight(uh, orc, enc, w)
+    y_ref = 0.5 * _ref(orc, enc, xb, enc_w).astype(np.float64)
+    r = torch.randn((m, n), generator=torch.Generator().manual_seed(3)).to(out)
+    y = r.clone().to(gpu)
+    lw.forward(x, y, residual=y, alpha=0.5)
+    assert_close(bf16_tensor_to_f32(y), y_ref + r.double().numpy(),
+                 bf16_out=out == torch.bfloat16, what=f"{enc} residual")
+    lg, enc_g = _weight(uh, orc, enc, w, gated=True)
+    p = 0.5 * _ref(orc, enc, xb, enc_g).astype(np.float64)
+    g, u = p[:, :n // 2], p[:, n // 2:]
+    yg = lg.forward(x, out_dtype=out, alpha=0.5)
+    assert_close(bf16_tensor_to_f32(yg), g / (1 + np.exp(-g)) * u,
+                 bf16_out=out == torch.bfloat16, what=f"{enc} gated")
+
+
+@pytest.mark.parametrize("enc", ["fp8", "aq4"])
+def test_wq_gemm_captured(uh, orc, gpu, enc):
+    """No scratch: workspace_size is 0, and a captured launch replays on new
+    inputs."""
+    m, n, k = 70, 528, 1024
+    lw, _ = _weight(uh, orc, enc, weights(n, k, tag=59))
+    assert lw.workspace_size(m) == 0
+    x = torch.zeros((m, k), dtype=torch.bfloat16, device=gpu)
+    y = torch.empty((m, n), dtype=torch.bfloat16, device=gpu)
+    s = torch.cuda.Stream()
+    with torch.cuda.stream(s):
+        lw.forward(x, y)
+        s.synchronize()
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph, stream=s):
+            lw.forward(x, y)
+    for i in range(3):
+        x.copy_(to_torch_bf16(activations_bf16(orc, m, k, tag=i + 430), gpu))
+        torch.cuda.synchronize()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(y, lw.forward(x))
+
+
+@pytest.mark.parametrize("enc", ["fp8", "aq4"])
+def test_wq_gemm_rows_are_independent(uh, orc, gpu, enc):
+    """A row of inf or NaN leaves the other rows' results as they are."""
+    for m, n in ((40, 300), (260, 2000)):
+        k = 512
+        lw, _ = _weight(uh, orc, enc, weights(n, k, tag=61))
+        x = to_torch_bf16(activations_bf16(orc, m, k, tag=440), gpu)
+        y = lw.forward(x)
+        x2 = x.clone()
+        x2[5, 17], x2[33, 100] = float("inf"), float("nan")
+        y2 = lw.forward(x2)
+        keep = torch.ones(m, dtype=torch.bool, device=gpu)
+        keep[5] = keep[33] = False
+        assert torch.equal(y[keep], y2[keep])
+        assert not torch.any(torch.isfinite(y2[33].float()))

@@ -25,7 +25,7 @@ BENCH_SOURCES = ["bench_read.hip", "check_bf16.hip"]
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 
 SOURCES = ["abi_v1.cpp", "linear_api.cpp", "safetensors.cpp", "evidence.hip", "noalloc.hip", "weights.hip",
-           "gemv.hip", "gemm_fp8.hip"]
+           "gemv.hip", "gemm_wq.hip", "gemm_fp8.hip"]
 
 COMMON = [
     "-O3", "-std=c++17", "-fPIC", "-fvisibility=hidden",

@@ -1,4 +1,5 @@
-// gemv.hip -- decode-shape (M <= 32 per pass) quantized GEMV on gfx950.
+// gemv.hip -- decode-shape (M <= 32 per pass) quantized GEMV on gfx950 (more
+// rows go to gemm_wq.hip, but for unaligned activations and ragged K).
 //
 // Y[m, n] = alpha * sum_k dequant(W)[n, k] * x[m, k], bf16 activations,
 // fp32 accumulation, for FP8-E4M3 per-row-scaled and AQ4 g128 weights.
@@ -2455,6 +2456,9 @@ hipError_t aq4_gemv_e(const GemvArgs &a, hipStream_t s) {
 
 // The epilogue kind is a template parameter of every kernel: dispatch once.
 hipError_t launch_fp8_gemv(const GemvArgs &a, hipStream_t s) {
+  if (const WqPlan p = plan_wq_gemm(a, false); p.taken) {
+    return launch_wq_gemm(a, false, p, s);
+  }
   switch (a.epi.kind) {
     case kEpiSiluMul: return fp8_gemv_e<kEpiSiluMul>(a, s);
     case kEpiResidual: return fp8_gemv_e<kEpiResidual>(a, s);
@@ -2463,6 +2467,9 @@ hipError_t launch_fp8_gemv(const GemvArgs &a, hipStream_t s) {
 }
 
 hipError_t launch_aq4_gemv(const GemvArgs &a, hipStream_t s) {
+  if (const WqPlan p = plan_wq_gemm(a, true); p.taken) {
+    return launch_wq_gemm(a, true, p, s);
+  }
   switch (a.epi.kind) {
     case kEpiSiluMul: return aq4_gemv_e<kEpiSiluMul>(a, s);
     case kEpiResidual: return aq4_gemv_e<kEpiResidual>(a, s);

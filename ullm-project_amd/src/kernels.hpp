@@ -66,6 +66,14 @@ struct GemvArgs {
 };
 hipError_t launch_fp8_gemv(const GemvArgs &a, hipStream_t s);
 hipError_t launch_aq4_gemv(const GemvArgs &a, hipStream_t s);
+// Blocks of a product of more than 32 rows (gemm_wq.hip; taken = false: the
+// decode kernels serve the call).
+struct WqPlan {
+  bool taken = false;
+  uint32_t cfg = 0, block_m = 0, block_n = 0, tiles = 0;
+};
+WqPlan plan_wq_gemm(const GemvArgs &a, bool aq4);
+hipError_t launch_wq_gemm(const GemvArgs &a, bool aq4, const WqPlan &p, hipStream_t s);
 // Bytes of split-K scratch the launch for these arguments would use (0: it
 // does not split).  The first bytes are counters that must be zero.
 uint64_t gemv_scratch_bytes(const GemvArgs &a, bool aq4);

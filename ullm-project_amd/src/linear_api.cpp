@@ -762,6 +762,13 @@ extern "C" ULLM_HIP_API ullm_status_t ullm_linear_forward_plan(
       a.k = static_cast<uint32_t>(w->k);
       a.n16 = static_cast<uint32_t>(fp8w ? w->fp8.n16 : w->aq4.n16);
       a.units = static_cast<uint32_t>(fp8w ? w->fp8.blocks_per_stripe() : w->aq4.groups);
+      if (const ullm::WqPlan p = ullm::plan_wq_gemm(a, !fp8w); p.taken) {
+        plan->kernel = ULLM_LINEAR_KERNEL_GEMM_LDS;
+        plan->block_m = p.block_m;
+        plan->block_n = p.block_n;
+        plan->tiles = plan->grid = p.tiles;
+        return ULLM_STATUS_OK;
+      }
       const ullm::GemvChoice c = ullm::gemv_choice(a, !fp8w, true);
       plan->kernel = ULLM_LINEAR_KERNEL_GEMV;
       plan->split_k = c.ks;
