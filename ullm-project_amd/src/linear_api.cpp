@@ -309,8 +309,7 @@ ullm_status_t create_weight(const ullm_linear_weight_desc_t *d,
   }
   HIP_TRY(sink, "hipMalloc (weight tiles)", hipMalloc(&w->tiles, w->tile_bytes));
   HIP_TRY(sink, "hipMalloc (weight scales)", hipMalloc(&w->aux, w->aux_bytes));
-  HIP_TRY(sink, "hipMemsetAsync", hipMemsetAsync(w->tiles, 0, w->tile_bytes, stream));
-  HIP_TRY(sink, "hipMemsetAsync", hipMemsetAsync(w->aux, 0, w->aux_bytes, stream));
+  // Every kernel below writes all of both buffers, padding included.
 
   DevBuf sv, ss, sz;
   const void *values = nullptr, *scales = nullptr, *zeros = nullptr;
