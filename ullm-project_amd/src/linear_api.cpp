@@ -84,7 +84,10 @@ class DeviceScope {
     if (hipGetDevice(&prev_) != hipSuccess) {
       prev_ = -1;
     }
-    err_ = hipSetDevice(device);
+    err_ = prev_ == device ? hipSuccess : hipSetDevice(device);
+    if (prev_ == device) {
+      prev_ = -1;  // nothing to restore
+    }
   }
   ~DeviceScope() {
     if (prev_ >= 0) {
