@@ -9,10 +9,10 @@
 // LDS (about 50 KB per microsecond and CU) at few.
 //
 // Two kernels, one choice (plan_wq_gemm):
-//   * wq_gemm_kernel: blocks of 32..256 rows x 128..256 columns, 8 waves
+//   * wq_gemm_kernel: blocks of 32..128 rows x 128..384 columns, 8 waves
 //     tiling the block, x staged in LDS for all of them.  MI355X, K = 4096,
-//     M = 2048, N = 28672: AQ4 1060 -> 490 us (0.98 PFLOP/s), FP8 1355 -> 450
-//     us (1.07 PFLOP/s); a plain bf16 GEMM of that size, weights already
+//     M = 2048, N = 28672: AQ4 1060 -> 447 us (1.08 PFLOP/s), FP8 1355 -> 414
+//     us (1.16 PFLOP/s); a plain bf16 GEMM of that size, weights already
 //     bf16, takes 407 us in the vendor's library.
 //   * wq_strip_kernel: blocks of 16..64 rows x 32..96 columns, the waves
 //     splitting K, each with an LDS ring of its own and no barrier before the
@@ -40,19 +40,22 @@ namespace {
 
 // Block configuration.  WM x WN waves of TM x TN 16 x 16 tiles; a k-step is
 // 128 k.  STAGES LDS stages of x, BD steps of weights in flight in registers,
-// a barrier every SPB steps.
+// a barrier every SPB steps.  WK = 2: two such groups of waves take the even
+// and the odd steps.
 template <uint32_t TM_, uint32_t TN_, uint32_t WM_, uint32_t WN_, uint32_t STAGES_,
-          uint32_t BD_ = 1, uint32_t SPB_ = 1>
+          uint32_t BD_ = 1, uint32_t SPB_ = 1, uint32_t WK_ = 1>
 struct WqCfg {
-  static constexpr uint32_t SPB = SPB_;
-  static_assert(STAGES_ % SPB == 0 && STAGES_ / SPB >= 2 && 4 % SPB == 0, "stages");
+  static constexpr uint32_t SPB = SPB_, WK = WK_;
+  static constexpr uint32_t G = SPB * WK;  // k-steps between barriers
+  static_assert(STAGES_ % G == 0 && STAGES_ / G >= 2 && 4 % SPB == 0, "stages");
+  static_assert(WK == 1 || (WK == 2 && TM_ % 2 == 0), "K groups");
   static constexpr uint32_t TM = TM_, TN = TN_, WM = WM_, WN = WN_, STAGES = STAGES_;
   static constexpr uint32_t BD = BD_;
-  static constexpr uint32_t WAVES = WM * WN;
+  static constexpr uint32_t WAVES = WM * WN * WK;
   static constexpr uint32_t BM = TM * WM * 16, BN = TN * WN * 16;
   static constexpr uint32_t A_BYTES = BM * 256;  // 128 k of every row
-  // AQ4 activation sums: two sets of four groups for every row.
-  static constexpr uint32_t XS_BYTES = 2 * BM * 16;
+  // AQ4 activation sums: two sets of four groups for every row (and WK).
+  static constexpr uint32_t XS_BYTES = WK * 2 * BM * 16;
   static constexpr uint32_t COPIES = BM / (4 * WAVES);
   static_assert(BM % (4 * WAVES) == 0 && WAVES % 4 == 0, "copy split");
   // Row pitch (bf16 elements) of a wave's epilogue chunk: 16 bytes of padding
@@ -116,11 +119,26 @@ __device__ __forceinline__ uint32_t wq_tile() {
 // (direct loads, whole 256-byte row segments, the 16-byte chunk c of row r at
 // slot c ^ (r % 16), so the 16 rows of an MFMA operand read hit 16 bank
 // groups), each wave loads its own TN weight tiles straight into registers,
-// unpacks them once and contracts them with its TM row tiles.  Every step's
-// products start from zero and are added to the fp32 accumulators per tile:
-// AQ4 needs that for the group scale (one multiply-add per element), FP8
-// keeps its sums as short as the decode kernels' (relative error 1.2e-7 at K
-// = 4096; one chain over K is 4 to 8 % faster and has 2.1e-7).
+// unpacks them once and contracts them with its TM row tiles.
+//
+// What bounds a step is the sum of its parts more than the largest: with the
+// copies taken out (timing only) the 256 x 192 block of two waves by four took
+// 434 of 504 us (M = 2048, N = 28672, AQ4), with the MFMAs taken out 206.  A
+// step costs each wave 4 TM TN MFMAs, an unpack of 32 (AQ4) or 16 (FP8) VALU
+// instructions per weight tile, 4 per product tile, and TM 4 KiB operand
+// reads.  All waves side by side over the columns (WM = 1) unpack every weight
+// once per block instead of once per WM: 128 x 256 blocks, 2 x 4 waves of
+// 64 x 64 against 1 x 8 of 128 x 32: FP8 2.01 -> 1.57 us per step, AQ4 1.87 ->
+// 1.79.  128 x 384 leaves the matrix cores the largest share (AQ4 447, FP8
+// 414 us, against 475 and 439 in 128 x 256).  64 x 128 blocks of one K group
+// read x from LDS as long as they contract it (16 columns per wave); with two
+// groups of four waves on alternating steps the reads halve (WK = 2: AQ4 M =
+// 512 14336 -> 4096 87 -> 75 us), at the price of an exchange at the end.
+//
+// Every step's products start from zero and are added to the fp32 accumulators
+// per tile: AQ4 needs that for the group scale (one multiply-add per element),
+// FP8 keeps its sums as short as the decode kernels' (relative error 1.2e-7 at
+// K = 4096; one chain over K is 4 to 8 % faster and has 2.1e-7).
 //
 // AQ4's sum_k x per (row, group): each of the WN waves that share a row tile
 // takes every WN-th one, sums it by an MFMA against ones and leaves it in
@@ -133,7 +151,8 @@ __global__ __launch_bounds__(C::WAVES *kWave) void wq_gemm_kernel(GemvArgs a) {
   extern __shared__ __attribute__((aligned(1024))) char lds[];
   const uint32_t lane = threadIdx.x % kWave;
   const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
-  const uint32_t wm = wave / C::WN, wn = wave % C::WN;
+  const uint32_t wk = wave / (C::WM * C::WN);  // 0 unless WK = 2
+  const uint32_t wm = wave / C::WN % C::WM, wn = wave % C::WN;
   const uint32_t stripes = a.n16 / 16;
   const uint32_t mblocks = (a.m + C::BM - 1) / C::BM;
   const uint32_t tile = wq_tile();
@@ -183,14 +202,16 @@ __global__ __launch_bounds__(C::WAVES *kWave) void wq_gemm_kernel(GemvArgs a) {
       }
     }
   };
-  // AQ4 scale|zero words of four groups: lane l holds group g0 + l / 16.
+  // Step u of this wave is k-step u WK + wk.
+  auto kstep = [&](uint32_t u) { return u * C::WK + wk; };
+  // AQ4 scale|zero words of four of its groups: lane l holds step u0 + l / 16.
   uint32_t zc[C::TN], zn[C::TN];
-  auto load_z = [&](uint32_t g0) {
+  auto load_z = [&](uint32_t u0) {
     if constexpr (AQ4) {
 #pragma unroll
       for (uint32_t j = 0; j < C::TN; ++j) {
-        zn[j] = __builtin_amdgcn_raw_buffer_load_b32(zbuf, lane * 4,
-                                                     (j * units + g0) * 64, 0);
+        zn[j] = __builtin_amdgcn_raw_buffer_load_b32(
+            zbuf, lane % 16 * 4 + lane / 16 * (C::WK * 64), (j * units + kstep(u0)) * 64, 0);
       }
     }
   };
@@ -203,14 +224,14 @@ __global__ __launch_bounds__(C::WAVES *kWave) void wq_gemm_kernel(GemvArgs a) {
       acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
     }
   }
-  float *xsb = reinterpret_cast<float *>(lds + C::MAIN_BYTES);
+  float *xsb = reinterpret_cast<float *>(lds + C::MAIN_BYTES) + wk * (2 * C::BM * 4);
   load_z(0);
 #pragma unroll
   for (uint32_t d = 0; d < C::BD; ++d) {
-    load_b(raw[d], d);
+    load_b(raw[d], kstep(d));
   }
 #pragma unroll
-  for (uint32_t t = 0; t + C::SPB < C::STAGES; ++t) {
+  for (uint32_t t = 0; t + C::G < C::STAGES; ++t) {
     copy_a(t, lds + t * C::A_BYTES);
   }
   const uint32_t nmask = opaque_u32(0x00780078u);
@@ -225,16 +246,16 @@ __global__ __launch_bounds__(C::WAVES *kWave) void wq_gemm_kernel(GemvArgs a) {
     const uint32_t c = AQ4 ? 4 * q + q4 : 8 * (q / 2) + 2 * q4 + q % 2;
     return *reinterpret_cast<const bf16x8 *>(st + arow + i * 4096 + ((c ^ sw) * 16));
   };
-  // acc -= sum over groups g0 .. g0 + 3 of (s (16 + z))[n] * xs[m], as one
-  // MFMA per tile: k-slots 8 q4 .. + 7 carry group g0 + q4's products of the
-  // three-way bf16 splits of both factors.
+  // acc -= sum over the groups of steps u0 .. u0 + 3 of (s (16 + z))[n] *
+  // xs[m], as one MFMA per tile: k-slots 8 q4 .. + 7 carry step u0 + q4's
+  // products of the three-way bf16 splits of both factors.
   auto split3 = [&](float v, float (&o)[3]) {
     o[0] = bits_f32(f32_bits(static_cast<float>(static_cast<__bf16>(v))));
     o[1] = static_cast<float>(static_cast<__bf16>(v - o[0]));
     o[2] = v - o[0] - o[1];
   };
-  auto correct = [&](uint32_t g0) {
-    const bool live = g0 + q4 < units;
+  auto correct = [&](uint32_t u0) {
+    const bool live = kstep(u0 + q4) < units;
     bf16x8 cb[C::TN];
 #pragma unroll
     for (uint32_t j = 0; j < C::TN; ++j) {
@@ -247,7 +268,7 @@ __global__ __launch_bounds__(C::WAVES *kWave) void wq_gemm_kernel(GemvArgs a) {
           bf16x8, u32x4{f32x2_to_bf16x2(o[0], o[1]), f32x2_to_bf16x2(o[0], o[1]),
                         f32x2_to_bf16x2(o[2], o[0]), f32x2_to_bf16x2(o[2], o[1])});
     }
-    const float *xold = xsb + ((g0 / 4) & 1) * (C::BM * 4) + q4;
+    const float *xold = xsb + ((u0 / 4) & 1) * (C::BM * 4) + q4;
 #pragma unroll
     for (uint32_t i = 0; i < C::TM; ++i) {
       float o[3];
@@ -264,16 +285,18 @@ __global__ __launch_bounds__(C::WAVES *kWave) void wq_gemm_kernel(GemvArgs a) {
   __builtin_amdgcn_s_waitcnt(0);
   wq_barrier();
 
-  uint32_t rd = 0, wr = C::STAGES - C::SPB;
-  // Step t (0..3) of the four that start at step g4.
-  // TAIL: the weights loaded ahead may be dead, so only the copies count as
-  // newer than the next step's.
-  auto step = [&](uint32_t g4, uint32_t t, auto tail) {
-    const uint32_t g = g4 + t;
-    const char *st = lds + rd * C::A_BYTES;
-    u32x4 (&rw)[C::TN][U] = raw[t % C::BD];
-    bf16x8 b[C::TN][4];
-    float sf[C::TN];
+  uint32_t rd = wk, wr = C::STAGES - C::G;
+  // Operands and scales of a step from its raw tiles (t: its place among the
+  // four of z).  The waves of a SIMD are a pair (w, w + WAVES / 2).  For AQ4
+  // the first unpacks a step at the end of the one before, the second at its
+  // own start, so that one's unpacking runs under the other's MFMAs (with
+  // both at the start: M = 512 14336 -> 4096 79.9 against 75.2 us, M = 2048
+  // 4096 -> 28672 in 128 x 256 blocks 503 against 483).  FP8's converts are
+  // half as many, and unpacking in two places spilled registers.
+  const bool late = !AQ4 || wave >= C::WAVES / 2;
+  bf16x8 b[C::TN][4];
+  float sf[C::TN];
+  auto unpack = [&](const u32x4 (&rw)[C::TN][U], const uint32_t (&z)[C::TN], uint32_t t) {
 #pragma unroll
     for (uint32_t j = 0; j < C::TN; ++j) {
       if constexpr (AQ4) {
@@ -282,7 +305,7 @@ __global__ __launch_bounds__(C::WAVES *kWave) void wq_gemm_kernel(GemvArgs a) {
           b[j][q] = nib8_to_bf16_off16(rw[j][0][q], nmask, nmagic);
         }
         sf[j] = f16_to_f32(uint16_t(
-            __builtin_amdgcn_ds_bpermute(int((t * 16 + sw) * 4), int(zc[j])) & 0xffff));
+            __builtin_amdgcn_ds_bpermute(int((t * 16 + sw) * 4), int(z[j])) & 0xffff));
       } else {
 #pragma unroll
         for (uint32_t u = 0; u < 2; ++u) {
@@ -290,18 +313,34 @@ __global__ __launch_bounds__(C::WAVES *kWave) void wq_gemm_kernel(GemvArgs a) {
         }
       }
     }
-    load_b(rw, g + C::BD);
+  };
+  if (!late) {
+    unpack(raw[0], zn, 0);
+  }
+  // This wave's step t (0..3) of the four that start at step u4.
+  // TAIL: the weights loaded ahead may be dead, so only the copies count as
+  // newer than the next step's.
+  auto step = [&](uint32_t u4, uint32_t t, auto tail) {
+    const uint32_t g = kstep(u4 + t);
+    const char *st = lds + rd * C::A_BYTES;
+    u32x4 (&rw)[C::TN][U] = raw[t % C::BD];
+    if (late) {
+      unpack(rw, zc, t);
+    }
+    load_b(rw, kstep(u4 + t + C::BD));
     if (t % C::SPB == 0) {
 #pragma unroll
-      for (uint32_t u = 0; u < C::SPB; ++u) {
-        copy_a(g + C::STAGES - C::SPB + u, lds + (wr + u) * C::A_BYTES);
+      for (uint32_t v = 0; v < C::G; ++v) {
+        copy_a((u4 + t) * C::WK + C::STAGES - C::G + v, lds + (wr + v) * C::A_BYTES);
       }
-      wr = wr + C::SPB == C::STAGES ? 0u : wr + C::SPB;
+      wr = wr + C::G == C::STAGES ? 0u : wr + C::G;
     }
     __builtin_amdgcn_sched_barrier(0);  // issued before any use below
     // An FP8 weight's K may end in the middle of its last step.
     const uint32_t nq = !AQ4 && decltype(tail)::value && units - g * 2 == 1 ? 2u : 4u;
-    float *xcur = xsb + ((g4 / 4) & 1) * (C::BM * 4) + t;
+    float *xcur = xsb + ((u4 / 4) & 1) * (C::BM * 4) + t;
+    // At the end one of two groups may have no step left.
+    if (C::WK == 1 || !decltype(tail)::value || g < steps) {
     bf16x8 av[4];
 #pragma unroll
     for (uint32_t q = 0; q < 4; ++q) {
@@ -348,45 +387,54 @@ __global__ __launch_bounds__(C::WAVES *kWave) void wq_gemm_kernel(GemvArgs a) {
       }
       __builtin_amdgcn_sched_barrier(0);
     }
-    rd = rd + 1 == C::STAGES ? 0u : rd + 1;
+    }
+    if (!late) {
+      unpack(raw[(t + 1) % C::BD], t == 3 ? zn : zc, (t + 1) % 4);
+    }
+    rd = rd + C::WK >= C::STAGES ? rd + C::WK - C::STAGES : rd + C::WK;
     // Every SPB steps: the next ones' copies have landed before the barrier;
     // later copies and weights stay in flight.
     if (t % C::SPB == C::SPB - 1) {
-      constexpr uint32_t R = C::STAGES / C::SPB;
-      constexpr uint32_t bl = decltype(tail)::value ? 0 : C::TN * U;
-      wq_wait_vm<(R - 2) * C::SPB * (C::COPIES + bl) + (C::SPB - 1) * bl>();
+      constexpr uint32_t R = C::STAGES / C::G;
+      constexpr uint32_t bl = decltype(tail)::value ? 0 : C::SPB * C::TN * U;
+      constexpr uint32_t last = decltype(tail)::value ? 0 : (C::SPB - 1) * C::TN * U;
+      wq_wait_vm<(R - 2) * (C::G * C::COPIES + bl) + last>();
       wq_barrier();
     }
   };
-  auto next_z = [&](uint32_t g4) {
+  auto next_z = [&](uint32_t u4) {
     if constexpr (AQ4) {
-      if (g4 != 0) {
-        correct(g4 - 4);
+      if (u4 != 0) {
+        correct(u4 - 4);
       }
 #pragma unroll
       for (uint32_t j = 0; j < C::TN; ++j) {
         zc[j] = zn[j];
       }
-      load_z(g4 + 4);
+      load_z(u4 + 4);
     }
   };
-  uint32_t g4 = 0;
+  uint32_t u4 = 0;
 #pragma clang loop unroll(disable)
-  for (; g4 + 4 <= steps; g4 += 4) {
-    next_z(g4);
+  for (; (u4 + 4) * C::WK <= steps; u4 += 4) {
+    next_z(u4);
 #pragma unroll
     for (uint32_t t = 0; t < 4; ++t) {
-      step(g4, t, std::false_type{});
+      step(u4, t, std::false_type{});
     }
   }
-  // The last one to three steps.
-  if (g4 < steps) {
-    next_z(g4);
-    step(g4, 0, std::true_type{});
-    if (g4 + 1 < steps) {
-      step(g4, 1, std::true_type{});
-      if (g4 + 2 < steps) {
-        step(g4, 2, std::true_type{});
+  // The last one to three steps (four of which one is short with WK = 2).
+  const uint32_t usteps = (steps + C::WK - 1) / C::WK;
+  if (u4 < usteps) {
+    next_z(u4);
+    step(u4, 0, std::true_type{});
+    if (u4 + 1 < usteps) {
+      step(u4, 1, std::true_type{});
+      if (u4 + 2 < usteps) {
+        step(u4, 2, std::true_type{});
+        if (C::WK > 1 && u4 + 3 < usteps) {
+          step(u4, 3, std::true_type{});
+        }
       }
     }
   }
@@ -395,8 +443,38 @@ __global__ __launch_bounds__(C::WAVES *kWave) void wq_gemm_kernel(GemvArgs a) {
 
   const uint32_t mw = m0 + wm * C::TM * 16 + 4 * q4;
   if constexpr (AQ4) {
-    correct((steps - 1) / 4 * 4);
-  } else {
+    correct((usteps - 1) / 4 * 4);
+  }
+  // The two K groups' sums: each wave hands the row tiles it will not store to
+  // the wave that will.
+  constexpr uint32_t HALF = C::TM / C::WK;
+  auto stores = [&](uint32_t i) { return C::WK == 1 || i / HALF == wk; };
+  if constexpr (C::WK > 1) {
+    static_assert(C::WAVES * HALF * C::TN * 1024 <= C::MAIN_BYTES, "exchange fits");
+    f32x4 *ex = reinterpret_cast<f32x4 *>(lds);
+    const uint32_t other = wave < C::WM * C::WN ? wave + C::WM * C::WN : wave - C::WM * C::WN;
+#pragma unroll
+    for (uint32_t i = 0; i < C::TM; ++i) {
+      if (!stores(i)) {
+#pragma unroll
+        for (uint32_t j = 0; j < C::TN; ++j) {
+          ex[((wave * HALF + i % HALF) * C::TN + j) * kWave + lane] = acc[i][j];
+        }
+      }
+    }
+    wq_barrier();
+#pragma unroll
+    for (uint32_t i = 0; i < C::TM; ++i) {
+      if (stores(i)) {
+#pragma unroll
+        for (uint32_t j = 0; j < C::TN; ++j) {
+          acc[i][j] += ex[((other * HALF + i % HALF) * C::TN + j) * kWave + lane];
+        }
+      }
+    }
+    wq_barrier();  // the chunks below reuse the exchange
+  }
+  if constexpr (!AQ4) {
     const float *scales = static_cast<const float *>(a.aux);
 #pragma unroll
     for (uint32_t j = 0; j < C::TN; ++j) {
@@ -414,6 +492,9 @@ __global__ __launch_bounds__(C::WAVES *kWave) void wq_gemm_kernel(GemvArgs a) {
   if (!vec) {
 #pragma unroll
     for (uint32_t i = 0; i < C::TM; ++i) {
+      if (!stores(i)) {
+        continue;
+      }
 #pragma unroll
       for (uint32_t j = 0; j < C::TN; ++j) {
 #pragma unroll
@@ -434,6 +515,9 @@ __global__ __launch_bounds__(C::WAVES *kWave) void wq_gemm_kernel(GemvArgs a) {
   const uint32_t n0 = T0 * tw, nlim = gated ? a.epi.n_out : a.n;
 #pragma unroll
   for (uint32_t i = 0; i < C::TM; ++i) {
+    if (!stores(i)) {
+      continue;
+    }
 #pragma unroll
     for (uint32_t j = 0; j < C::TN; ++j) {
       float v[4];
@@ -750,11 +834,11 @@ hipError_t launch_strip_t(const GemvArgs &a, hipStream_t s) {
   return hipGetLastError();
 }
 
-using W256x192 = WqCfg<8, 3, 2, 4, 2>;
-using W192x256 = WqCfg<6, 4, 2, 4, 3>;
-using W128x256 = WqCfg<4, 4, 2, 4, 3>;
+using W128x384 = WqCfg<8, 3, 1, 8, 3>;
+using W128x256 = WqCfg<8, 2, 1, 8, 3>;
 using W64x128 = WqCfg<4, 1, 1, 8, 4, 2, 2>;
 using W32x128 = WqCfg<2, 1, 1, 8, 6, 2, 2>;
+using W64x128K = WqCfg<4, 2, 1, 4, 6, 2, 1, 2>;
 using S64x64 = StripCfg<4, 4, 4>;
 using S48x64 = StripCfg<3, 4, 6>;
 using S48x48 = StripCfg<3, 3, 6>;
@@ -770,46 +854,46 @@ using S16x32 = StripCfg<1, 2, 8>;
 // Fitted to launches of every configuration on one MI355X (256 CUs, weights
 // from HBM) over M = 33 .. 2048 and (N, K) = (1024 | 4096 | 6144 | 14336 |
 // 28672, 4096), (4096, 14336), (2560, 1024), (9000, 2048).  The choice it
-// makes is the fastest of the 13 or within 1 % of it on average, 12 % at
+// makes is the fastest of the 13 or within 1 % of it on average, 10 % at
 // worst; without the 48-row strips it is up to 18 % worse (M = 64, N = 6144),
-// with fewer row heights of the 8-wave blocks up to 23 % (M = 384, N = 28672:
-// 192 rows against 256).
+// without the 64 x 128 blocks of one K group up to 14 % (M = 384, N = 9000).
 struct WqCost {
   uint32_t bm, bn;
   float aq4[3], fp8[3];  // t0, step, tile; t0 < 0: not used
 };
 constexpr WqCost kWqCosts[] = {
-    {256, 192, {0.00f, 2.804f, 4.90f}, {0.00f, 2.486f, 3.55f}},
-    {192, 256, {0.00f, 2.729f, 5.26f}, {-1.0f, 0.0f, 0.0f}},
-    {128, 256, {0.00f, 1.985f, 4.28f}, {0.00f, 2.011f, 1.91f}},
-    {64, 128, {3.61f, 0.647f, 0.00f}, {3.05f, 0.574f, 0.01f}},
-    {32, 128, {3.55f, 0.413f, 0.00f}, {2.68f, 0.371f, 0.08f}},
-    {64, 64, {0.61f, 0.347f, 4.74f}, {0.62f, 0.314f, 4.50f}},
-    {48, 64, {1.06f, 0.280f, 4.22f}, {1.42f, 0.279f, 3.42f}},
-    {48, 48, {1.25f, 0.234f, 3.44f}, {1.36f, 0.240f, 3.08f}},
-    {32, 96, {4.34f, 0.274f, 1.02f}, {3.53f, 0.254f, 1.36f}},
-    {32, 64, {3.39f, 0.215f, 0.64f}, {2.61f, 0.208f, 0.91f}},
-    {32, 48, {3.02f, 0.168f, 0.68f}, {2.34f, 0.170f, 0.91f}},
-    {32, 32, {2.77f, 0.144f, 0.34f}, {2.08f, 0.152f, 0.53f}},
-    {16, 32, {2.51f, 0.078f, 0.59f}, {2.33f, 0.095f, 0.64f}},
+    {128, 384, {0.00f, 2.374f, 6.04f}, {0.00f, 2.155f, 5.00f}},
+    {128, 256, {0.00f, 1.788f, 4.37f}, {0.00f, 1.593f, 3.51f}},
+    {64, 128, {3.71f, 0.671f, 0.00f}, {2.92f, 0.588f, 0.00f}},
+    {64, 128, {0.23f, 0.612f, 3.60f}, {-1.0f, 0.0f, 0.0f}},
+    {32, 128, {3.57f, 0.416f, 0.00f}, {2.64f, 0.376f, 0.05f}},
+    {64, 64, {0.65f, 0.344f, 4.72f}, {0.58f, 0.314f, 4.52f}},
+    {48, 64, {1.11f, 0.280f, 4.16f}, {1.40f, 0.282f, 3.39f}},
+    {48, 48, {1.27f, 0.233f, 3.41f}, {1.35f, 0.241f, 3.07f}},
+    {32, 96, {4.27f, 0.275f, 1.04f}, {3.51f, 0.255f, 1.36f}},
+    {32, 64, {3.35f, 0.214f, 0.62f}, {2.63f, 0.209f, 0.88f}},
+    {32, 48, {3.03f, 0.169f, 0.65f}, {2.36f, 0.171f, 0.88f}},
+    {32, 32, {2.73f, 0.143f, 0.33f}, {2.07f, 0.151f, 0.53f}},
+    {16, 32, {2.46f, 0.078f, 0.58f}, {2.30f, 0.095f, 0.64f}},
 };
 enum : uint32_t {
-  kW256x192, kW192x256, kW128x256, kW64x128, kW32x128, kS64x64, kS48x64,
+  kW128x384, kW128x256, kW64x128, kW64x128K, kW32x128, kS64x64, kS48x64,
   kS48x48, kS32x96, kS32x64, kS32x48, kS32x32, kS16x32
 };
 
 template <bool AQ4, int EPI>
 hipError_t wq_e(const GemvArgs &a, uint32_t cfg, hipStream_t s) {
   switch (cfg) {
-    case kW256x192: return launch_wq_t<AQ4, W256x192, EPI>(a, s);
-    case kW192x256:
-      // FP8 spills registers in this block and never takes it.
-      if constexpr (AQ4) {
-        return launch_wq_t<AQ4, W192x256, EPI>(a, s);
-      }
-      break;
+    case kW128x384: return launch_wq_t<AQ4, W128x384, EPI>(a, s);
     case kW128x256: return launch_wq_t<AQ4, W128x256, EPI>(a, s);
     case kW64x128: return launch_wq_t<AQ4, W64x128, EPI>(a, s);
+    case kW64x128K:
+      // FP8 gains on one round only (M = 512 14336 -> 4096 79 against 72 us)
+      // and loses on more.
+      if constexpr (AQ4) {
+        return launch_wq_t<AQ4, W64x128K, EPI>(a, s);
+      }
+      break;
     case kW32x128: return launch_wq_t<AQ4, W32x128, EPI>(a, s);
     case kS64x64: return launch_strip_t<AQ4, S64x64, EPI>(a, s);
     case kS48x64: return launch_strip_t<AQ4, S48x64, EPI>(a, s);
