@@ -219,6 +219,8 @@ struct GemmCfg {
   // (M=2048 N=8192).
   static constexpr bool EARLY_SCALES = PP && BM < 256;
   static_assert(LDS <= 160 * 1024, "gfx950 LDS per workgroup");
+  // Blocks a K split may use; those of even_fill are planned unsplit only.
+  static constexpr bool SPLITS = PP && BM != 192 && !(BM == 128 && BN == 192);
 };
 
 // Zero scale operands: the compiler emits the unscaled
@@ -936,6 +938,11 @@ using GemmSmall128 = GemmCfg<128, 64, 4, 2, 3, 3, true>;
 using GemmSmall64 = GemmCfg<64, 64, 2, 4, 3, 3, true>;
 using GemmSmall128W = GemmCfg<128, 128, 2, 4, 3, 3, true>;
 using GemmSmall64W = GemmCfg<64, 128, 2, 4, 3, 3, true>;
+// 192 x 128, 128 x 192 and 192 x 192: one-round grids the 256-row blocks
+// leave part empty (even_fill); waves of 48 x 64, 64 x 48 and 96 x 48.
+using GemmEven128x192 = GemmCfg<128, 192, 2, 4, 3, 3, true>;
+using GemmEven192x128 = GemmCfg<192, 128, 4, 2, 3, 3, true>;
+using GemmEven192x192 = GemmCfg<192, 192, 2, 4, 3, 3, true>;
 
 
 // Block width (256, 224 or 192 columns, 256 rows) whose rounds of
@@ -1143,7 +1150,7 @@ hipError_t raise_lds_limit(const void *kernel, uint32_t bytes) {
 template <class C, uint32_t EPI>
 hipError_t launch_gemm_lds(const GemmArgs &a, const GemmPlan &p,
                            hipStream_t s) {
-  if constexpr (C::PP) {
+  if constexpr (C::SPLITS) {
     if (p.ksplit > 1) {
       const void *ks = reinterpret_cast<const void *>(fp8_gemm_lds_kernel<C, EPI, true>);
       const hipError_t attr = raise_lds_limit(ks, C::LDS);
@@ -1178,6 +1185,9 @@ hipError_t gemm_e(const GemmArgs &a, const GemmPlan &p, bool vec,
     case kGemmSmall64: return launch_gemm_lds<GemmSmall64, EPI>(a, p, s);
     case kGemmSmall128W: return launch_gemm_lds<GemmSmall128W, EPI>(a, p, s);
     case kGemmSmall64W: return launch_gemm_lds<GemmSmall64W, EPI>(a, p, s);
+    case kGemmEven128x192: return launch_gemm_lds<GemmEven128x192, EPI>(a, p, s);
+    case kGemmEven192x128: return launch_gemm_lds<GemmEven192x128, EPI>(a, p, s);
+    case kGemmEven192x192: return launch_gemm_lds<GemmEven192x192, EPI>(a, p, s);
     case kGemmLarge: return launch_gemm_lds<GemmLarge, EPI>(a, p, s);
     default: break;
   }
@@ -1186,15 +1196,13 @@ hipError_t gemm_e(const GemmArgs &a, const GemmPlan &p, bool vec,
   return hipGetLastError();
 }
 
-}  // namespace
-
 // The LDS kernel serves every M (rows past M are clamped on load and masked
 // on store): at K = 4096 it is 24 us against the direct kernel's 39 us for
 // M = 32..96, N = 4096, and 30 against 55-60 us at N = 28672.  The direct
 // kernel takes unaligned activations, K not a multiple of 128, and offsets
 // past 32 bits.
-GemmPlan plan_fp8_gemm(uint32_t m, uint32_t n, uint32_t k, bool vec,
-                       bool offsets_fit, uint32_t cus) {
+GemmPlan plan_wide(uint32_t m, uint32_t n, uint32_t k, bool vec,
+                   bool offsets_fit, uint32_t cus) {
   GemmPlan p{};
   p.ksplit = 1;
   if (!(vec && offsets_fit && k % 128 == 0)) {
@@ -1208,7 +1216,8 @@ GemmPlan plan_fp8_gemm(uint32_t m, uint32_t n, uint32_t k, bool vec,
   // Tuning overrides (read only by a -DULLM_TUNING build): ULLM_GEMM_CFG=mid,
   // ULLM_GEMM_BN=256/224/192/128/64, ULLM_GEMM_BM=256/128/64 (rows of the 64-
   // and 128-column blocks), ULLM_GEMM_PERSIST=0 (one workgroup per tile),
-  // ULLM_GEMM_SPLIT=0 and ULLM_GEMM_SPLIT_STEPS (the K split).
+  // ULLM_GEMM_SPLIT=0 and ULLM_GEMM_SPLIT_STEPS (the K split) and
+  // ULLM_GEMM_EVEN=0 (no blocks of 192 by 128 or 192).
   const char *cfg = tuning_env("ULLM_GEMM_CFG");
   const char *bn_env = tuning_env("ULLM_GEMM_BN");
   const char *persist_env = tuning_env("ULLM_GEMM_PERSIST");
@@ -1249,6 +1258,55 @@ GemmPlan plan_fp8_gemm(uint32_t m, uint32_t n, uint32_t k, bool vec,
     default: p.kind = kGemmLarge; fill_plan<GemmLarge>(p, m, n, cus, persist); break;
   }
   plan_split(p, k, cus);
+  return p;
+}
+
+// Blocks of 192 rows or columns in place of a one-round, unsplit grid of
+// 256-row blocks that leaves CUs idle or pads rows.  On such grids a
+// workgroup's time is its copies (block rows + columns per k-step), so the
+// smaller block wins where its grid still needs one round only.  Measured on
+// MI355X, weights from HBM (old against new, us):
+// - 192 x 128 for 256 x 128, at every K: M=777 N=6144 K=128 6.3 / 5.5, K=1024
+//   12.1 / 10.0, K=4096 32.8 / 28.4; M=1536 N=4096 K=4096 32.6 / 28.5,
+//   K=14336 97.5 / 87.3; M=300 N=14336 33.2 / 28.1; M=157 N=19312 K=2048
+//   19.6 / 16.8.
+// - 192 x 128 for 256 x 64, half the tiles at the same copies each, once the
+//   256 x 64 grid fills most of the CUs and K is long enough: M=512 N=8192
+//   K=4096 29.6 / 26.2, M=1024 N=4000 K=2048 15.9 / 14.3, K=512 7.4 / 7.4;
+//   at 144 to 168 tiles it lost 1-4 %.
+// - 128 x 192 for 256 x 128 where 192 x 128 needs two rounds: M=1024 N=6144
+//   K=4096 32.8 / 29.7, K=1024 12.0 / 11.8, K=512 8.9 / 9.3; M=215 N=22512
+//   K=7168, of fewer copied rows, 59.5 / 60.4.
+// - 192 x 192 for 256 x 192: M=750 N=12288 K=4096 43.3 / 39.2, K=1024 17.0 /
+//   16.9, K=512 11.2 / 12.7; M=709 N=11024 K=1536 22.3 / 18.9.
+void even_fill(GemmPlan &p, uint32_t m, uint32_t n, uint32_t k, uint32_t cus) {
+  const char *env = tuning_env("ULLM_GEMM_EVEN");
+  if (p.ksplit > 1 || p.grid < p.tiles || (env != nullptr && env[0] == '0')) {
+    return;
+  }
+  const auto one_round = [&](uint64_t bm, uint64_t bn) {
+    return ((m + bm - 1) / bm) * ((n + bn - 1) / bn) <= cus;
+  };
+  const bool longk = k >= 1024;
+  if (one_round(192, 128) && (p.kind == kGemmNarrow128 ||
+                              (p.kind == kGemmNarrow64 && longk && p.tiles * 32 > cus * 25))) {
+    p.kind = kGemmEven192x128;
+    fill_plan<GemmEven192x128>(p, m, n, cus, false);
+  } else if (one_round(128, 192) && p.kind == kGemmNarrow128 && longk && m > 224) {
+    p.kind = kGemmEven128x192;
+    fill_plan<GemmEven128x192>(p, m, n, cus, false);
+  } else if (one_round(192, 192) && p.kind == kGemmNarrow192 && longk) {
+    p.kind = kGemmEven192x192;
+    fill_plan<GemmEven192x192>(p, m, n, cus, false);
+  }
+}
+
+}  // namespace
+
+GemmPlan plan_fp8_gemm(uint32_t m, uint32_t n, uint32_t k, bool vec,
+                       bool offsets_fit, uint32_t cus) {
+  GemmPlan p = plan_wide(m, n, k, vec, offsets_fit, cus);
+  even_fill(p, m, n, k, cus);
   return p;
 }
 

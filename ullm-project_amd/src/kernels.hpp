@@ -105,6 +105,9 @@ enum GemmKind : uint32_t {
   kGemmSmall64 = 8,     // LDS-pipelined 64 x 64 (short prompts)
   kGemmSmall128W = 9,   // LDS-pipelined 128 x 128 (short prompts)
   kGemmSmall64W = 10,   // LDS-pipelined 64 x 128 (short prompts)
+  kGemmEven128x192 = 11,  // LDS-pipelined 128 x 192
+  kGemmEven192x128 = 12,  // LDS-pipelined 192 x 128
+  kGemmEven192x192 = 13,  // LDS-pipelined 192 x 192
 };
 struct GemmPlan {
   uint32_t kind, block_m, block_n, tiles, grid;
