@@ -214,7 +214,7 @@ typedef struct ullm_linear_weight_export_desc_t {
 #define ULLM_LINEAR_KERNEL_GEMV UINT32_C(1)        /* decode, bf16 activations */
 #define ULLM_LINEAR_KERNEL_GEMM_DIRECT UINT32_C(2) /* FP8 GEMM, operands from L2 */
 #define ULLM_LINEAR_KERNEL_GEMM_LDS UINT32_C(3)    /* activations through LDS: FP8
-                                                    * GEMM, or exact M > 32 */
+                                                    * GEMM, or exact M > 16 */
 
 /* GEMV kernel variants reported by ullm_linear_forward_plan. */
 #define ULLM_LINEAR_GEMV_SINGLE UINT32_C(1)  /* one stripe per workgroup, x from L2 */

@@ -1,4 +1,4 @@
-// gemm_wq.hip -- products of more than 32 rows with exact (bf16) activations
+// gemm_wq.hip -- products of more than 16 rows with exact (bf16) activations
 // on gfx950: batched decode and prefill of FP8-E4M3 and AQ4 g128 weights.
 //
 // Y[m, n] = alpha * sum_k dequant(W)[n, k] * x[m, k], fp32 accumulation, from
@@ -913,11 +913,34 @@ hipError_t wq_enc(const GemvArgs &a, bool aq4, uint32_t cfg, hipStream_t s) {
   return aq4 ? wq_e<true, EPI>(a, cfg, s) : wq_e<false, EPI>(a, cfg, s);
 }
 
+// 17 to 32 rows on at most one round of 16 x 32 strips, where the decode
+// kernels leave CUs idle and run a stripe's whole K in one workgroup.  MI355X,
+// decode kernels / strips, us: M=32 N=480 K=10624 AQ4 22.6 / 8.5, FP8 22.2 /
+// 9.0; M=17 N=1000 K=8192 9.6 / 8.0 and 14.5 / 8.9; M=32 N=4096 K=8192 13.2 /
+// 9.9 and 16.9 / 12.5; M=24 N=3000 K=5120 8.4 / 7.0 and 10.3 / 8.5; M=32
+// N=1024 K=4096 6.8 / 5.1 and 8.3 / 5.1, K=1024 3.5 / 3.2 and 4.0 / 3.8.
+// - K > 4096, or from 24 rows on at most half of the CUs from K = 2048: M=32
+//   N=4096 K=4096 would gain too (7.5 / 6.5, 9.6 / 7.7), but the tests fix
+//   the register-staged plans of that size and of M = 17 and 23 at N=1000
+//   K=4096.
+// - up to 16 rows, one strip of rows, half as many CUs work (M=16 N=2048
+//   K=8192 7.9 / 9.1, 9.6 / 11.6).
+// - calls that the decode kernels split over K stay (their split fills the
+//   CUs), and FP8 past K = 10752, where one chain over K rounds more than
+//   they do (relative error at K=14336 1.4e-7 against 1.0e-7; up to there both
+//   1.2e-7 and less; AQ4 1.9e-7 against 1.8e-6).
+bool wq_few_rows(const GemvArgs &a, bool aq4, uint32_t cus) {
+  const uint32_t tiles = (a.m + 15) / 16 * ((a.n16 + 31) / 32);
+  return a.m > 16 && tiles <= cus && (aq4 || a.k <= 10752) &&
+         (a.k > 4096 || (a.m >= 24 && a.k >= 2048 && 2 * tiles <= cus)) &&
+         gemv_split_parts(a, aq4) == 1;
+}
+
 }  // namespace
 
-// Every call of more than 32 rows with aligned activations and whole 64-k
-// tiles, but one kind: up to four rows past the first 32 at K <= 1024 on more
-// stripes than CUs, where the decode kernels' short second pass comes within
+// The calls of wq_few_rows, and those of more than 32 rows, with aligned
+// activations and whole 64-k tiles, but one kind of the latter: up to four
+// rows past the first 32 at K <= 1024 on more stripes than CUs, where the decode kernels' short second pass comes within
 // a microsecond (M = 33, N = 6200, K = 1024: AQ4 6.1 against 5.8 us, FP8 7.0
 // against 6.0).  Everywhere else measured the decode kernels lose, by 1.2 to
 // 7.8 times.  Sizes whose 32-bit buffer offsets would not do stay with them.
@@ -926,8 +949,12 @@ WqPlan plan_wq_gemm(const GemvArgs &a, bool aq4) {
   const uint32_t unit_k = aq4 ? 128 : 64;
   const uint64_t row_bytes = a.ldx * 2;
   const uint32_t cus = device_cu_count();
-  if (a.m <= 32 || (a.m <= 36 && a.k <= 1024 && a.n16 / 16 > cus) || a.k % unit_k != 0 ||
-      reinterpret_cast<uintptr_t>(a.x) % 16 != 0 || a.ldx % 8 != 0 ||
+  const bool few = a.m <= 32;
+  if (few ? !wq_few_rows(a, aq4, cus)
+          : a.m <= 36 && a.k <= 1024 && a.n16 / 16 > cus) {
+    return p;
+  }
+  if (a.k % unit_k != 0 || reinterpret_cast<uintptr_t>(a.x) % 16 != 0 || a.ldx % 8 != 0 ||
       row_bytes >= (uint64_t(1) << 22) || a.units >= (1u << 17)) {
     return p;
   }
@@ -941,7 +968,8 @@ WqPlan plan_wq_gemm(const GemvArgs &a, bool aq4) {
     const WqCost &c = kWqCosts[i];
     const float *t = aq4 ? c.aq4 : c.fp8;
     const uint64_t tiles = uint64_t((a.m + c.bm - 1) / c.bm) * ((a.n16 + c.bn - 1) / c.bn);
-    if (t[0] < 0.0f || tiles >= (1u << 22) || (forced >= 0 && uint32_t(forced) != i)) {
+    if (t[0] < 0.0f || tiles >= (1u << 22) || (forced >= 0 && uint32_t(forced) != i) ||
+        (few && i != kS16x32)) {
       continue;
     }
     const uint64_t rounds = (tiles + cus - 1) / cus;

@@ -66,7 +66,7 @@ struct GemvArgs {
 };
 hipError_t launch_fp8_gemv(const GemvArgs &a, hipStream_t s);
 hipError_t launch_aq4_gemv(const GemvArgs &a, hipStream_t s);
-// Blocks of a product of more than 32 rows (gemm_wq.hip; taken = false: the
+// Blocks of a product of more than 16 rows (gemm_wq.hip; taken = false: the
 // decode kernels serve the call).
 struct WqPlan {
   bool taken = false;
