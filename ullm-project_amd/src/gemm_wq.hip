@@ -741,6 +741,31 @@ __global__ __launch_bounds__(C::WAVES *kWave) void wq_strip_kernel(GemvArgs a) {
   for (uint32_t r = 0; r + 1 < C::DEPTH; ++r) {
     issue(ring[r], sb + r, r);
   }
+  // FP8: the chain of a wave's products is cut every DEPTH steps and the parts
+  // are added up: relative error at M=64 N=4096 K=14336 1.0e-7 instead of
+  // 2.0e-7 (the decode kernels 1.4e-7), M=203 N=5003 K=4096 8.0e-8 instead of
+  // 1.1e-7 (9.1e-8), at the same time (26.7 / 26.5 us, 21.5 / 21.7).
+  f32x4 sum[C::TM][C::TN];
+  if constexpr (!AQ4) {
+#pragma unroll
+    for (uint32_t i = 0; i < C::TM; ++i) {
+#pragma unroll
+      for (uint32_t j = 0; j < C::TN; ++j) {
+        sum[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+      }
+    }
+  }
+  auto fold = [&]() {
+#pragma unroll
+    for (uint32_t i = 0; i < C::TM; ++i) {
+#pragma unroll
+      for (uint32_t j = 0; j < C::TN; ++j) {
+        sum[i][j] += acc[i][j];
+        acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+        asm volatile("" : "+v"(sum[i][j]));
+      }
+    }
+  };
   const uint32_t n = se - sb;
   for (uint32_t t = 0; t < n; t += C::DEPTH) {
 #pragma unroll
@@ -757,6 +782,9 @@ __global__ __launch_bounds__(C::WAVES *kWave) void wq_strip_kernel(GemvArgs a) {
       }
       asm volatile("" ::: "memory");
     }
+    if constexpr (!AQ4) {
+      fold();
+    }
   }
   wq_wait_vm<0>();
   asm volatile("" ::: "memory");
@@ -766,7 +794,7 @@ __global__ __launch_bounds__(C::WAVES *kWave) void wq_strip_kernel(GemvArgs a) {
   for (uint32_t i = 0; i < C::TM; ++i) {
 #pragma unroll
     for (uint32_t j = 0; j < C::TN; ++j) {
-      red[(i * C::TN + j) * kWave + lane] = acc[i][j];
+      red[(i * C::TN + j) * kWave + lane] = AQ4 ? acc[i][j] : sum[i][j];
     }
   }
   wq_barrier();
@@ -926,9 +954,9 @@ hipError_t wq_enc(const GemvArgs &a, bool aq4, uint32_t cfg, hipStream_t s) {
 // - up to 16 rows, one strip of rows, half as many CUs work (M=16 N=2048
 //   K=8192 7.9 / 9.1, 9.6 / 11.6).
 // - calls that the decode kernels split over K stay (their split fills the
-//   CUs), and FP8 past K = 10752, where one chain over K rounds more than
-//   they do (relative error at K=14336 1.4e-7 against 1.0e-7; up to there both
-//   1.2e-7 and less; AQ4 1.9e-7 against 1.8e-6).
+//   CUs), and FP8 past K = 10752, the longest K measured unsplit at these
+//   sizes.  Relative error at K = 10624: FP8 9.2e-8 against 1.3e-7, AQ4 1.9e-7
+//   against 1.8e-6.
 bool wq_few_rows(const GemvArgs &a, bool aq4, uint32_t cus) {
   const uint32_t tiles = (a.m + 15) / 16 * ((a.n16 + 31) / 32);
   return a.m > 16 && tiles <= cus && (aq4 || a.k <= 10752) &&
