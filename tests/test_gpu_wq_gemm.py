@@ -122,6 +122,46 @@ def test_wq_gemm_parity(uh, orc, gpu, enc, m, n, k):
     assert_close(bf16_tensor_to_f32(yb), y_ref, bf16_out=True, what=f"{enc} bf16 {m}x{n}x{k}")
 
 
+# FP8 K of 8 i + 7 tiles of 64: a whole number of four-step rounds whose last
+# step is half one.  (m, n, k) for each block of 8 waves.
+HALF_STEPS = [
+    ((32, 128), 37, 6564, 448), ((32, 128), 40, 8250, 960), ((32, 128), 34, 8255, 1472),
+    ((32, 128), 65, 8314, 4032),
+    ((64, 128), 37, 17140, 448), ((64, 128), 37, 17117, 960), ((64, 128), 35, 16407, 1472),
+    ((64, 128), 40, 19069, 4032),
+    ((128, 256), 129, 26336, 448), ((128, 256), 129, 26171, 960), ((128, 256), 130, 26261, 1472),
+    ((128, 256), 129, 26266, 4032),
+    ((128, 384), 259, 26239, 448), ((128, 384), 258, 26363, 960), ((128, 384), 257, 21942, 1472),
+    ((128, 384), 257, 22039, 4032),
+]
+
+
+@pytest.mark.parametrize("block,m,n,k", HALF_STEPS)
+def test_wq_gemm_half_last_step(uh, orc, gpu, block, m, n, k):
+    """Nothing past K counts: not the next stripe's weights, and neither the
+    columns beside a strided x nor the next row (both NaN or inf here)."""
+    lw, enc_w = _weight(uh, orc, "fp8", weights(n, k, tag=63))
+    xb = activations_bf16(orc, m, k, tag=m + 450)
+    rows = np.unique(np.r_[0, 4, 15, 31, 32, np.arange(0, m, 37), m - 2, m - 1])
+    y_ref = _ref(orc, "fp8", np.ascontiguousarray(xb[rows]), enc_w)
+    x = to_torch_bf16(xb, gpu)
+    wide = torch.full((m, k + 64), float("nan"), dtype=torch.bfloat16, device=gpu)
+    wide[:, :k] = x
+    y = torch.full((m, n), float("nan"), device=gpu)
+    _block(lw, x, y, block)
+    lw.forward(x, y)
+    # The bound of test_wq_gemm_parity.
+    rel = max(1e-5, 8 * 2.0 ** -24 * k ** 0.5)
+    assert_close(y[rows].cpu().numpy(), y_ref, rel=rel, what=f"{block} {m}x{n}x{k}")
+    assert torch.equal(lw.forward(wide[:, :k], out_dtype=torch.float32), y)
+    bad = x.clone()
+    bad[5], bad[33] = float("nan"), float("inf")
+    y2 = lw.forward(bad, out_dtype=torch.float32)
+    keep = torch.ones(m, dtype=torch.bool, device=gpu)
+    keep[5] = keep[33] = False
+    assert torch.equal(y2[keep], y[keep])
+
+
 @pytest.mark.parametrize("m,n", [(50, 1100), (300, 2056)])
 @pytest.mark.parametrize("enc", ["fp8", "aq4"])
 def test_wq_gemm_strided_and_unaligned(uh, orc, gpu, enc, m, n):

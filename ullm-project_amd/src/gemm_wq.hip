@@ -414,16 +414,20 @@ __global__ __launch_bounds__(C::WAVES *kWave) void wq_gemm_kernel(GemvArgs a) {
       load_z(u4 + 4);
     }
   };
+  // Whole steps only: an FP8 weight's half step, which ends at an odd number of
+  // 64-k tiles, must find its tail step below whatever the count is.
+  const uint32_t whole = units / U;
   uint32_t u4 = 0;
 #pragma clang loop unroll(disable)
-  for (; (u4 + 4) * C::WK <= steps; u4 += 4) {
+  for (; (u4 + 4) * C::WK <= whole; u4 += 4) {
     next_z(u4);
 #pragma unroll
     for (uint32_t t = 0; t < 4; ++t) {
       step(u4, t, std::false_type{});
     }
   }
-  // The last one to three steps (four of which one is short with WK = 2).
+  // The last one to three steps (four where the last is an FP8 half step, or
+  // where one of two groups has none).
   const uint32_t usteps = (steps + C::WK - 1) / C::WK;
   if (u4 < usteps) {
     next_z(u4);
@@ -432,7 +436,7 @@ __global__ __launch_bounds__(C::WAVES *kWave) void wq_gemm_kernel(GemvArgs a) {
       step(u4, 1, std::true_type{});
       if (u4 + 2 < usteps) {
         step(u4, 2, std::true_type{});
-        if (C::WK > 1 && u4 + 3 < usteps) {
+        if ((!AQ4 || C::WK > 1) && u4 + 3 < usteps) {
           step(u4, 3, std::true_type{});
         }
       }
