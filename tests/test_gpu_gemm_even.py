@@ -21,13 +21,16 @@ CASES = [
     ("192x128", 777, 6144, 128),     # one k-step, last row block of 9 rows
     ("192x128", 768, 6130, 256),     # whole row blocks, ragged N
     ("192x128", 157, 19304, 384),    # one row block, part of it past M
-    ("192x128", 193, 15000, 1152),   # from 256 x 64; last row block of 1 row
+    ("192x128", 385, 10800, 1152),   # last row block of 1 row, ragged N
     ("128x192", 1000, 6100, 1024),   # ragged both ways
     ("192x192", 750, 12200, 1152),   # ragged both ways
 ]
 # The neighbours of the rule's lines keep their blocks.
 KEPT = [
     ("256x64", 1024, 4000, 128), ("256x64", 420, 4592, 1152),
+    # 200 to 256 tiles of 256 x 64, which 192 x 128 blocks do not beat
+    ("256x64", 193, 15000, 1152), ("256x64", 240, 14336, 4096), ("256x64", 512, 8192, 1024),
+    ("256x64", 1024, 4096, 4096),
     ("256x128", 1000, 6144, 512), ("256x128", 215, 22512, 1024),
     ("256x192", 750, 12288, 512), ("256x128", 2048, 4096, 1024),
 ]

@@ -1270,10 +1270,11 @@ GemmPlan plan_wide(uint32_t m, uint32_t n, uint32_t k, bool vec,
 //   12.1 / 10.0, K=4096 32.8 / 28.4; M=1536 N=4096 K=4096 32.6 / 28.5,
 //   K=14336 97.5 / 87.3; M=300 N=14336 33.2 / 28.1; M=157 N=19312 K=2048
 //   19.6 / 16.8.
-// - 192 x 128 for 256 x 64, half the tiles at the same copies each, once the
-//   256 x 64 grid fills most of the CUs and K is long enough: M=512 N=8192
-//   K=4096 29.6 / 26.2, M=1024 N=4000 K=2048 15.9 / 14.3, K=512 7.4 / 7.4;
-//   at 144 to 168 tiles it lost 1-4 %.
+// - not for 256 x 64, whose workgroups copy no more than 192 x 128 ones and
+//   spread over twice as many CUs: at 200 to 256 of its tiles 192 x 128 lost
+//   nearly everywhere, M=193 N=14720 K=4096 25.5 / 28.9, M=384 N=6528 K=12032
+//   58.6 / 65.0, M=1024 N=4096 K=12032 65.7 / 71.4, K=1152 10.0 / 10.4, M=512
+//   N=8192 K=4096 26.2 / 26.2.
 // - 128 x 192 for 256 x 128 where 192 x 128 needs two rounds: M=1024 N=6144
 //   K=4096 32.8 / 29.7, K=1024 12.0 / 11.8, K=512 8.9 / 9.3; M=215 N=22512
 //   K=7168, of fewer copied rows, 59.5 / 60.4.
@@ -1288,8 +1289,7 @@ void even_fill(GemmPlan &p, uint32_t m, uint32_t n, uint32_t k, uint32_t cus) {
     return ((m + bm - 1) / bm) * ((n + bn - 1) / bn) <= cus;
   };
   const bool longk = k >= 1024;
-  if (one_round(192, 128) && (p.kind == kGemmNarrow128 ||
-                              (p.kind == kGemmNarrow64 && longk && p.tiles * 32 > cus * 25))) {
+  if (one_round(192, 128) && p.kind == kGemmNarrow128) {
     p.kind = kGemmEven192x128;
     fill_plan<GemmEven192x128>(p, m, n, cus, false);
   } else if (one_round(128, 192) && p.kind == kGemmNarrow128 && longk && m > 224) {
