@@ -11,8 +11,8 @@
 // Two kernels, one choice (plan_wq_gemm):
 //   * wq_gemm_kernel: blocks of 32..128 rows x 128..384 columns, 8 waves
 //     tiling the block, x staged in LDS for all of them.  MI355X, K = 4096,
-//     M = 2048, N = 28672: AQ4 1060 -> 447 us (1.08 PFLOP/s), FP8 1355 -> 414
-//     us (1.16 PFLOP/s); a plain bf16 GEMM of that size, weights already
+//     M = 2048, N = 28672: AQ4 1060 -> 447 us (1.08 PFLOP/s), FP8 1350 -> 433
+//     us (1.11 PFLOP/s); a plain bf16 GEMM of that size, weights already
 //     bf16, takes 407 us in the vendor's library.
 //   * wq_strip_kernel: blocks of 16..64 rows x 32..96 columns, the waves
 //     splitting K, each with an LDS ring of its own and no barrier before the
@@ -129,16 +129,23 @@ __device__ __forceinline__ uint32_t wq_tile() {
 // reads.  All waves side by side over the columns (WM = 1) unpack every weight
 // once per block instead of once per WM: 128 x 256 blocks, 2 x 4 waves of
 // 64 x 64 against 1 x 8 of 128 x 32: FP8 2.01 -> 1.57 us per step, AQ4 1.87 ->
-// 1.79.  128 x 384 leaves the matrix cores the largest share (AQ4 447, FP8
-// 414 us, against 475 and 439 in 128 x 256).  64 x 128 blocks of one K group
+// 1.79.  128 x 384 leaves the matrix cores the largest share (AQ4 447 us
+// against 475 in 128 x 256).  64 x 128 blocks of one K group
 // read x from LDS as long as they contract it (16 columns per wave); with two
 // groups of four waves on alternating steps the reads halve (WK = 2: AQ4 M =
 // 512 14336 -> 4096 87 -> 75 us), at the price of an exchange at the end.
 //
 // Every step's products start from zero and are added to the fp32 accumulators
-// per tile: AQ4 needs that for the group scale (one multiply-add per element),
-// FP8 keeps its sums as short as the decode kernels' (relative error 1.2e-7 at
-// K = 4096; one chain over K is 4 to 8 % faster and has 2.1e-7).
+// per tile: AQ4 needs that for the group scale (one multiply-add per element).
+// FP8 adds them up in two levels, four steps and then these sums, which keeps
+// the error below the decode kernels' (relative, against 64-bit sums; decode
+// kernels / one level / two, K = 4096 9.0e-8 / 1.15e-7 / 7.9e-8, K = 14336
+// 1.45e-7 / 1.98e-7 / 1.14e-7) in the same time (128 x 256 and 64 x 128 within
+// 3 %): the first step of four starts the sum, so a round makes as many
+// additions as before.  The second set of sums fits 128 x 256 blocks (228
+// registers); in 128 x 384 ones it spills 253, so FP8 does without them (M =
+// 2048 N = 28672 433 us against 414, M = 1463 N = 7214 K = 6848, one round
+// there and two here, 186 against 131).
 //
 // AQ4's sum_k x per (row, group): each of the WN waves that share a row tile
 // takes every WN-th one, sums it by an MFMA against ones and leaves it in
@@ -317,6 +324,24 @@ __global__ __launch_bounds__(C::WAVES *kWave) void wq_gemm_kernel(GemvArgs a) {
   if (!late) {
     unpack(raw[0], zn, 0);
   }
+  // FP8's second level of sums: every four steps' sum is added to the total.
+  f32x4 sum[AQ4 ? 1 : C::TM][AQ4 ? 1 : C::TN];
+  if constexpr (!AQ4) {
+    static_assert(AQ4 || C::WK == 1, "a round's first step is its wave's own");
+#pragma unroll
+    for (uint32_t i = 0; i < C::TM; ++i) {
+#pragma unroll
+      for (uint32_t j = 0; j < C::TN; ++j) {
+        sum[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+      }
+    }
+  }
+  auto fold = [&](uint32_t i, uint32_t j) {
+    if constexpr (!AQ4) {
+      sum[i][j] += acc[i][j];
+      asm volatile("" : "+v"(sum[i][j]));
+    }
+  };
   // This wave's step t (0..3) of the four that start at step u4.
   // TAIL: the weights loaded ahead may be dead, so only the copies count as
   // newer than the next step's.
@@ -378,12 +403,16 @@ __global__ __launch_bounds__(C::WAVES *kWave) void wq_gemm_kernel(GemvArgs a) {
       for (uint32_t j = 0; j < C::TN; ++j) {
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
-          acc[i][j][r] = AQ4 ? __builtin_fmaf(sf[j], p[j][r], acc[i][j][r])
-                             : acc[i][j][r] + p[j][r];
+          acc[i][j][r] = AQ4      ? __builtin_fmaf(sf[j], p[j][r], acc[i][j][r])
+                         : t == 0 ? p[j][r]
+                                  : acc[i][j][r] + p[j][r];
         }
         // Keeps the sums here: sunk below the next row tile's branch they
         // would keep every tile's products alive.
         asm volatile("" : "+v"(acc[i][j]));
+        if (!AQ4 && t == 3) {
+          fold(i, j);
+        }
       }
       __builtin_amdgcn_sched_barrier(0);
     }
@@ -439,6 +468,16 @@ __global__ __launch_bounds__(C::WAVES *kWave) void wq_gemm_kernel(GemvArgs a) {
         if ((!AQ4 || C::WK > 1) && u4 + 3 < usteps) {
           step(u4, 3, std::true_type{});
         }
+      }
+    }
+  }
+  if constexpr (!AQ4) {
+    const bool open = usteps % 4 != 0;  // the last round ended before its fourth step
+#pragma unroll
+    for (uint32_t i = 0; i < C::TM; ++i) {
+#pragma unroll
+      for (uint32_t j = 0; j < C::TN; ++j) {
+        acc[i][j] = open ? sum[i][j] + acc[i][j] : sum[i][j];
       }
     }
   }
@@ -886,7 +925,7 @@ using S16x32 = StripCfg<1, 2, 8>;
 // Fitted to launches of every configuration on one MI355X (256 CUs, weights
 // from HBM) over M = 33 .. 2048 and (N, K) = (1024 | 4096 | 6144 | 14336 |
 // 28672, 4096), (4096, 14336), (2560, 1024), (9000, 2048).  The choice it
-// makes is the fastest of the 13 or within 1 % of it on average, 10 % at
+// makes is the fastest of the table or within 1 % of it on average, 10 % at
 // worst; without the 48-row strips it is up to 18 % worse (M = 64, N = 6144),
 // without the 64 x 128 blocks of one K group up to 14 % (M = 384, N = 9000).
 struct WqCost {
@@ -894,7 +933,7 @@ struct WqCost {
   float aq4[3], fp8[3];  // t0, step, tile; t0 < 0: not used
 };
 constexpr WqCost kWqCosts[] = {
-    {128, 384, {0.00f, 2.374f, 6.04f}, {0.00f, 2.155f, 5.00f}},
+    {128, 384, {0.00f, 2.374f, 6.04f}, {-1.0f, 0.0f, 0.0f}},
     {128, 256, {0.00f, 1.788f, 4.37f}, {0.00f, 1.593f, 3.51f}},
     {64, 128, {3.71f, 0.671f, 0.00f}, {2.92f, 0.588f, 0.00f}},
     {64, 128, {0.23f, 0.612f, 3.60f}, {-1.0f, 0.0f, 0.0f}},
@@ -916,7 +955,12 @@ enum : uint32_t {
 template <bool AQ4, int EPI>
 hipError_t wq_e(const GemvArgs &a, uint32_t cfg, hipStream_t s) {
   switch (cfg) {
-    case kW128x384: return launch_wq_t<AQ4, W128x384, EPI>(a, s);
+    case kW128x384:
+      // FP8's two levels of sums do not fit its registers.
+      if constexpr (AQ4) {
+        return launch_wq_t<AQ4, W128x384, EPI>(a, s);
+      }
+      break;
     case kW128x256: return launch_wq_t<AQ4, W128x256, EPI>(a, s);
     case kW64x128: return launch_wq_t<AQ4, W64x128, EPI>(a, s);
     case kW64x128K:
