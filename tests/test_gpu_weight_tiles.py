@@ -86,3 +86,15 @@ def test_fp8_rows_off_the_plain_encode(uh, orc, gpu):
     q, s = lw.export()
     assert np.array_equal(_bits(s), _bits(s_ref))
     assert np.array_equal(q, q_ref)
+
+
+@pytest.mark.parametrize("n,k,gated", [(16, 128, False), (15, 384, False), (4096, 1024, False),
+                                       (18, 256, True), (1000, 4096, True)])
+def test_device_bytes(uh, gpu, n, k, gated):
+    """A weight holds its padded rows once: half a byte (AQ4) or a byte (FP8)
+    per element, and a scale|zero word per group or a scale per row."""
+    n16 = 2 * -(-(n // 2) // 8) * 8 if gated else -(-n // 16) * 16
+    w = torch.zeros((n, k), device=gpu)
+    for enc, expect in ((uh.ENCODING_AQ4_G128, n16 * k // 2 + n16 * (k // 128) * 4),
+                        (uh.ENCODING_FP8_E4M3_ROW, n16 * k + n16 * 4)):
+        assert uh.LinearWeight.quantize(w, enc, gated=gated).info().device_bytes == expect

@@ -70,7 +70,7 @@ struct Aq4Layout {
   uint64_t n, k, n16, groups;
   uint64_t gate;  // F of a gated-pair weight, 0 for a plain one
   __host__ __device__ uint64_t phys(uint64_t row) const { return phys_row(row, gate); }
-  __host__ __device__ uint64_t words() const { return n16 * groups * 256; }
+  __host__ __device__ uint64_t words() const { return n16 / 16 * groups * 256; }
   __host__ __device__ uint64_t sz_words() const { return n16 * groups; }
 };
 

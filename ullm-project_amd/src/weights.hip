@@ -42,9 +42,9 @@ __device__ float block_max(float v, float *red) {
 // tile's place in the matrix a wave-uniform division instead of one per
 // element.  They are bound by memory.  Padding rows and columns
 // are written as zeros, so the buffers need no clearing first.  MI355X, N =
-// 14336, K = 4096 (element-wise kernels with byte or word accesses before):
-// FP8 quantize 183 -> 76 us and decode 136 -> 50 us, AQ4 quantize 116 -> 82
-// us and decode 128 -> 73 us.
+// 14336, K = 4096, sources from HBM (element-wise kernels with byte or word
+// accesses before): FP8 quantize 174 -> 61 us and decode 162 -> 55 us, AQ4
+// quantize 118 -> 50 us and decode 127 -> 59 us.
 
 // Calls f(tile index, stripe, unit) for each of this wave's tiles (of
 // stripes x units; more than one only past kMaxTileBlocks workgroups).
