@@ -1126,27 +1126,6 @@ void fill_plan(GemmPlan &p, uint32_t m, uint32_t n, uint32_t cus,
   p.grid = persist && p.tiles > slots ? slots : p.tiles;
 }
 
-// Dynamic-LDS limit of a kernel raised once per (kernel, device).
-hipError_t raise_lds_limit(const void *kernel, uint32_t bytes) {
-  static std::mutex mu;
-  static std::set<std::pair<const void *, int>> done;
-  int dev = 0;
-  hipError_t e = hipGetDevice(&dev);
-  if (e != hipSuccess) {
-    return e;
-  }
-  std::lock_guard<std::mutex> lock(mu);
-  if (done.count({kernel, dev}) != 0) {
-    return hipSuccess;
-  }
-  e = hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize,
-                          int(bytes));
-  if (e == hipSuccess) {
-    done.insert({kernel, dev});
-  }
-  return e;
-}
-
 template <class C, uint32_t EPI>
 hipError_t launch_gemm_lds(const GemmArgs &a, const GemmPlan &p,
                            hipStream_t s) {
@@ -1302,6 +1281,26 @@ void even_fill(GemmPlan &p, uint32_t m, uint32_t n, uint32_t k, uint32_t cus) {
 }
 
 }  // namespace
+
+hipError_t raise_lds_limit(const void *kernel, uint32_t bytes) {
+  static std::mutex mu;
+  static std::set<std::pair<const void *, int>> done;
+  int dev = 0;
+  hipError_t e = hipGetDevice(&dev);
+  if (e != hipSuccess) {
+    return e;
+  }
+  std::lock_guard<std::mutex> lock(mu);
+  if (done.count({kernel, dev}) != 0) {
+    return hipSuccess;
+  }
+  e = hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize,
+                          int(bytes));
+  if (e == hipSuccess) {
+    done.insert({kernel, dev});
+  }
+  return e;
+}
 
 GemmPlan plan_fp8_gemm(uint32_t m, uint32_t n, uint32_t k, bool vec,
                        bool offsets_fit, uint32_t cus) {

@@ -27,10 +27,7 @@
 // 8-wave blocks) and 2e-7 (the strips) against the decode kernels' 1.8e-6.
 #include <algorithm>
 #include <cstdlib>
-#include <mutex>
-#include <set>
 #include <type_traits>
-#include <utility>
 
 #include "device_common.hpp"
 #include "kernels.hpp"
@@ -859,30 +856,10 @@ __global__ __launch_bounds__(C::WAVES *kWave) void wq_strip_kernel(GemvArgs a) {
   }
 }
 
-
-hipError_t raise_lds(const void *kernel, uint32_t bytes) {
-  static std::mutex mu;
-  static std::set<std::pair<const void *, int>> done;
-  int dev = 0;
-  hipError_t e = hipGetDevice(&dev);
-  if (e != hipSuccess) {
-    return e;
-  }
-  std::lock_guard<std::mutex> lock(mu);
-  if (done.count({kernel, dev}) != 0) {
-    return hipSuccess;
-  }
-  e = hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, int(bytes));
-  if (e == hipSuccess) {
-    done.insert({kernel, dev});
-  }
-  return e;
-}
-
 template <bool AQ4, class C, int EPI>
 hipError_t launch_wq_t(const GemvArgs &a, hipStream_t s) {
   const void *k = reinterpret_cast<const void *>(wq_gemm_kernel<AQ4, C, EPI>);
-  const hipError_t e = raise_lds(k, C::LDS);
+  const hipError_t e = raise_lds_limit(k, C::LDS);
   if (e != hipSuccess) {
     return e;
   }
@@ -895,7 +872,7 @@ hipError_t launch_wq_t(const GemvArgs &a, hipStream_t s) {
 template <bool AQ4, class C, int EPI>
 hipError_t launch_strip_t(const GemvArgs &a, hipStream_t s) {
   const void *k = reinterpret_cast<const void *>(wq_strip_kernel<AQ4, C, EPI>);
-  const hipError_t e = raise_lds(k, C::LDS);
+  const hipError_t e = raise_lds_limit(k, C::LDS);
   if (e != hipSuccess) {
     return e;
   }

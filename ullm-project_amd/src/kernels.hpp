@@ -148,6 +148,8 @@ ullm_status_t forward_dispatch(const ullm_linear_forward_desc_t *desc,
 
 // Compute units of the current device, looked up once per device.
 uint32_t device_cu_count();
+// Raises a kernel's dynamic-LDS limit, once per (kernel, current device).
+hipError_t raise_lds_limit(const void *kernel, uint32_t bytes);
 // Launch-plan overrides for tuning sweeps.  Only a library built with
 // -DULLM_TUNING reads them from the environment; the default build returns
 // null for every name, so the launchers always take the configurations the
