@@ -154,13 +154,6 @@ __device__ __forceinline__ float wave_max(float v) {
   }
   return v;
 }
-__device__ __forceinline__ float wave_min(float v) {
-#pragma unroll
-  for (int off = 32; off > 0; off >>= 1) {
-    v = fminf(v, __shfl_xor(v, off, kWave));
-  }
-  return v;
-}
 
 // Byte-range buffer over device memory: loads at offsets past `bytes` return
 // zero without a memory access, which lets a software pipeline issue its

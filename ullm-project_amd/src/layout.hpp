@@ -50,26 +50,45 @@ __host__ __device__ constexpr uint64_t phys_row(uint64_t n, uint64_t gate) {
 __host__ __device__ constexpr uint64_t phys_rows(uint64_t n, uint64_t gate) {
   return gate == 0 ? round_up(n, 16) : 2 * round_up(gate, 8);
 }
+// Canonical row stored at physical row p of a weight of n rows (>= n:
+// padding), the inverse of phys_row.
+__host__ __device__ constexpr uint64_t canonical_row(uint64_t p, uint64_t n, uint64_t gate) {
+  if (gate == 0) {
+    return p;
+  }
+  const uint64_t f = p / 16 * 8 + p % 8;
+  return f >= gate ? n : p % 16 < 8 ? f : gate + f;
+}
+
+// Every row of a weight comes back from its place, and no other place holds one.
+constexpr bool rows_invert(uint64_t n, uint64_t gate) {
+  uint64_t live = 0;
+  for (uint64_t p = 0; p < phys_rows(n, gate); ++p) {
+    live += canonical_row(p, n, gate) < n ? 1 : 0;
+  }
+  for (uint64_t r = 0; r < n; ++r) {
+    const uint64_t p = phys_row(r, gate);
+    if (p >= phys_rows(n, gate) || canonical_row(p, n, gate) != r) {
+      return false;
+    }
+  }
+  return live == n;
+}
+static_assert(rows_invert(1, 0) && rows_invert(16, 0) && rows_invert(37, 0), "plain rows");
+static_assert(rows_invert(2, 1) && rows_invert(16, 8) && rows_invert(32, 16) &&
+                  rows_invert(26, 13) && rows_invert(62, 31),
+              "gated-pair rows");
 
 struct Fp8Layout {
   uint64_t n, k, n16, k64;
   uint64_t gate;  // F of a gated-pair weight, 0 for a plain one
-  __host__ __device__ uint64_t phys(uint64_t row) const { return phys_row(row, gate); }
   __host__ __device__ uint64_t blocks_per_stripe() const { return k64 / 64; }
   __host__ __device__ uint64_t bytes() const { return n16 * k64; }
-  // Byte of canonical element (row, col).
-  __host__ __device__ uint64_t offset(uint64_t row, uint64_t col) const {
-    row = phys(row);
-    const uint64_t lane = (row % 16) + 16 * ((col % 64) / 16);
-    return (((row / 16) * blocks_per_stripe() + col / 64) * 64 + lane) * 16 +
-           col % 16;
-  }
 };
 
 struct Aq4Layout {
   uint64_t n, k, n16, groups;
   uint64_t gate;  // F of a gated-pair weight, 0 for a plain one
-  __host__ __device__ uint64_t phys(uint64_t row) const { return phys_row(row, gate); }
   __host__ __device__ uint64_t words() const { return n16 / 16 * groups * 256; }
   __host__ __device__ uint64_t sz_words() const { return n16 * groups; }
 };

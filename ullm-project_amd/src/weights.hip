@@ -58,16 +58,6 @@ __device__ __forceinline__ void for_tiles(uint64_t stripes, uint64_t units, F f)
   }
 }
 
-// Canonical row stored at physical row p (>= n: padding), the inverse of
-// phys_row().
-__device__ __forceinline__ uint64_t canonical_row(uint64_t p, uint64_t n, uint64_t gate) {
-  if (gate == 0) {
-    return p;
-  }
-  const uint64_t f = p / 16 * 8 + p % 8;
-  return f >= gate ? n : p % 16 < 8 ? f : gate + f;
-}
-
 __device__ __forceinline__ bool aligned16(const void *p) {
   return reinterpret_cast<uintptr_t>(p) % 16 == 0;
 }
