@@ -208,6 +208,8 @@ def test_wq_gemm_strided_and_unaligned(uh, orc, gpu, enc, m, n):
     for dt in (torch.bfloat16, torch.float32):
         buf = torch.full((m, n + 5), 7.0, dtype=dt, device=gpu)
         y = buf[:, 3:3 + n]
+        _block(lw, wide[:, 8:8 + k], y, (32, 128) if m > 64 else
+               (32, 32) if enc == "fp8" else (16, 32))
         lw.forward(wide[:, 8:8 + k], y)
         assert_close(bf16_tensor_to_f32(y.contiguous()), y_ref, bf16_out=dt == torch.bfloat16,
                      what=f"{enc} strided")
@@ -228,6 +230,7 @@ def test_wq_gemm_epilogues(uh, orc, gpu, enc, m, n, out):
     y_ref = 0.5 * _ref(orc, enc, xb, enc_w).astype(np.float64)
     r = torch.randn((m, n), generator=torch.Generator().manual_seed(3)).to(out)
     y = r.clone().to(gpu)
+    _block(lw, x, y, (32, 128) if m > 64 else (32, 32) if enc == "fp8" else (16, 32))
     lw.forward(x, y, residual=y, alpha=0.5)
     assert_close(bf16_tensor_to_f32(y), y_ref + r.double().numpy(),
                  bf16_out=out == torch.bfloat16, what=f"{enc} residual")
@@ -237,6 +240,48 @@ def test_wq_gemm_epilogues(uh, orc, gpu, enc, m, n, out):
     yg = lg.forward(x, out_dtype=out, alpha=0.5)
     assert_close(bf16_tensor_to_f32(yg), g / (1 + np.exp(-g)) * u,
                  bf16_out=out == torch.bfloat16, what=f"{enc} gated")
+
+
+# (encoding, block, m, n, k) with rows of 16-byte segments (N and F multiples
+# of 8) and part of the last block past M and past N.
+SEGMENTS = [
+    ("fp8", (32, 128), 300, 2064, 384), ("aq4", (32, 128), 300, 2064, 384),
+    ("fp8", (64, 128), 65, 11072, 256), ("aq4", (64, 128), 129, 20000, 640),
+    ("aq4", (64, 128), 100, 12000, 640),  # two groups of waves over K
+    ("fp8", (128, 256), 200, 24688, 384), ("aq4", (128, 256), 200, 24688, 384),
+    ("aq4", (128, 384), 321, 27280, 384),
+]
+
+
+@pytest.mark.parametrize("epi", ["none", "silu", "residual"])
+@pytest.mark.parametrize("enc,block,m,n,k", SEGMENTS)
+def test_wq_gemm_segment_stores(uh, orc, gpu, enc, block, m, n, k, epi):
+    """The 8-wave blocks' bf16 rows leave in 16-byte segments, whole and cut at
+    the edges: the same bits as the fp32 output rounded, which is held to the
+    oracle on sampled rows, and nothing written beside them."""
+    lw, enc_w = _weight(uh, orc, enc, weights(n, k, tag=65), gated=epi == "silu")
+    xb = activations_bf16(orc, m, k, tag=m + 460)
+    rows = np.unique(np.r_[0, 15, 16, 31, 32, np.arange(0, m, 41), m - 1].clip(0, m - 1))
+    ref = 0.5 * _ref(orc, enc, np.ascontiguousarray(xb[rows]), enc_w).astype(np.float64)
+    x = to_torch_bf16(xb, gpu)
+    cols = n
+    if epi == "silu":
+        cols = n // 2
+        ref = ref[:, :cols] / (1 + np.exp(-ref[:, :cols])) * ref[:, cols:]
+    buf = torch.full((m + 1, cols + 8), 7.0, dtype=torch.bfloat16, device=gpu)
+    y = buf[:m, :cols]
+    y32 = torch.full((m, cols), float("nan"), device=gpu)
+    kw, kw32 = {}, {}
+    if epi == "residual":
+        y.copy_(torch.randn((m, n), generator=torch.Generator().manual_seed(m)))
+        kw, kw32 = {"residual": y}, {"residual": y.float()}
+        ref = ref + y[rows].double().cpu().numpy()
+    _block(lw, x, y, block)
+    lw.forward(x, y32, alpha=0.5, **kw32)
+    lw.forward(x, y, alpha=0.5, **kw)
+    assert_close(y32[rows].cpu().numpy(), ref, what=f"{enc} {block} {epi}")
+    assert torch.equal(y, y32.to(torch.bfloat16))
+    assert torch.all(buf[:, cols:] == 7.0) and torch.all(buf[m] == 7.0)
 
 
 @pytest.mark.parametrize("enc", ["fp8", "aq4"])
