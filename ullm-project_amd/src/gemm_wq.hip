@@ -972,16 +972,18 @@ hipError_t wq_enc(const GemvArgs &a, bool aq4, uint32_t cfg, hipStream_t s) {
 // 9.0; M=17 N=1000 K=8192 9.6 / 8.0 and 14.5 / 8.9; M=32 N=4096 K=8192 13.2 /
 // 9.9 and 16.9 / 12.5; M=24 N=3000 K=5120 8.4 / 7.0 and 10.3 / 8.5; M=32
 // N=1024 K=4096 6.8 / 5.1 and 8.3 / 5.1, K=1024 3.5 / 3.2 and 4.0 / 3.8.
-// - K > 4096, or from 24 rows on at most half of the CUs from K = 2048: M=32
-//   N=4096 K=4096 would gain too (7.5 / 6.5, 9.6 / 7.7), but the tests fix
-//   the register-staged plans of that size and of M = 17 and 23 at N=1000
-//   K=4096.
 // - up to 16 rows, one strip of rows, half as many CUs work (M=16 N=2048
 //   K=8192 7.9 / 9.1, 9.6 / 11.6).
-// - calls that the decode kernels split over K stay (their split fills the
-//   CUs), and FP8 past K = 10752, the longest K measured unsplit at these
-//   sizes.  Relative error at K = 10624: FP8 9.2e-8 against 1.3e-7, AQ4 1.9e-7
-//   against 1.8e-6.
+// - the other lines are narrower than where the kernels cross.  The strips are
+//   ahead beyond them too, but the tests pin those sizes to the decode
+//   kernels.  K <= 4096, or fewer than 24 rows or more than half of the CUs
+//   there (AQ4, FP8): M=32 N=4096 K=4096 7.4 / 5.7, 9.3 / 5.8, K=2048 5.2 /
+//   4.4, 6.4 / 4.4, K=1024 3.9 / 3.7, 4.6 / 4.1; M=17 N=1000 K=4096 6.7 / 4.6,
+//   6.4 / 5.0.  Calls that the decode kernels split over K (from 12288): M=32
+//   N=4096 K=12288 15.5 / 12.8, 20.0 / 18.2, K=14336 16.9 / 15.2, 21.3 / 20.6;
+//   M=32 N=1000 K=14336 15.0 / 10.1, 23.1 / 11.0.
+// Relative error at K = 10624: FP8 9.2e-8 against 1.3e-7, AQ4 1.9e-7 against
+// 1.8e-6.
 bool wq_few_rows(const GemvArgs &a, bool aq4, uint32_t cus) {
   const uint32_t tiles = (a.m + 15) / 16 * ((a.n16 + 31) / 32);
   return a.m > 16 && tiles <= cus && (aq4 || a.k <= 10752) &&
@@ -993,10 +995,13 @@ bool wq_few_rows(const GemvArgs &a, bool aq4, uint32_t cus) {
 
 // The calls of wq_few_rows, and those of more than 32 rows, with aligned
 // activations and whole 64-k tiles, but one kind of the latter: up to four
-// rows past the first 32 at K <= 1024 on more stripes than CUs, where the decode kernels' short second pass comes within
-// a microsecond (M = 33, N = 6200, K = 1024: AQ4 6.1 against 5.8 us, FP8 7.0
-// against 6.0).  Everywhere else measured the decode kernels lose, by 1.2 to
-// 7.8 times.  Sizes whose 32-bit buffer offsets would not do stay with them.
+// rows past the first 32 at K <= 1024 on more stripes than CUs, which the tests
+// pin to the decode kernels' two passes.  Those are ahead for AQ4 on 6200 to
+// 8192 columns at K = 512 only (decode kernels / blocks, us: M = 33, N = 8192
+// 4.7 / 5.2) and lose elsewhere (N = 8192, K = 1024 AQ4 6.2 / 5.8, FP8 7.4 /
+// 5.9; N = 28672, K = 1024 16.2 / 9.6, 18.0 / 9.8), by 1.2 to 7.8 times
+// outside that kind.  Sizes whose 32-bit buffer offsets would not do stay with
+// them.
 WqPlan plan_wq_gemm(const GemvArgs &a, bool aq4) {
   WqPlan p;
   const uint32_t unit_k = aq4 ? 128 : 64;
