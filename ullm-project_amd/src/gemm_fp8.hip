@@ -1250,8 +1250,8 @@ GemmPlan plan_wide(uint32_t m, uint32_t n, uint32_t k, bool vec,
 //   K=14336 97.5 / 87.3; M=300 N=14336 33.2 / 28.1; M=157 N=19312 K=2048
 //   19.6 / 16.8.
 // - not for 256 x 64, whose workgroups copy no more than 192 x 128 ones and
-//   spread over twice as many CUs: at 200 to 256 of its tiles 192 x 128 lost
-//   nearly everywhere, M=193 N=14720 K=4096 25.5 / 28.9, M=384 N=6528 K=12032
+//   fill as many CUs or up to twice as many: at 204 to 256 of its tiles 192 x
+//   128 lost nearly everywhere, M=193 N=14720 K=4096 25.5 / 28.9, M=384 N=6528 K=12032
 //   58.6 / 65.0, M=1024 N=4096 K=12032 65.7 / 71.4, K=1152 10.0 / 10.4, M=512
 //   N=8192 K=4096 26.2 / 26.2.
 // - 128 x 192 for 256 x 128 where 192 x 128 needs two rounds: M=1024 N=6144
